@@ -49,7 +49,9 @@ typedef struct mbir_ctx mbir_ctx;
 typedef struct mbir_job mbir_job;
 
 /* Context options (no reference counterpart: device selection and the HBM
- * budget used for admission by the batch/serve paths). */
+ * budget used for admission by the batch/serve paths).  Between calls a context keeps at
+ * most 64 MiB of device scratch and 16 MiB of pinned host memory, until it and its last job
+ * are closed; a server gives the scratch back where its budget has no room for it. */
 typedef struct mbir_opts {
   int32_t device;            /* HIP device ordinal */
   int32_t verbose;           /* 0 quiet, 1 progress lines on stderr */

@@ -184,6 +184,16 @@ hipError_t mbir_pool::device_alloc(void** p, size_t bytes)
   return r;
 }
 
+void mbir_pool::trim(size_t room)
+{
+  std::unique_lock<std::mutex> lk(scratch_mu, std::try_to_lock);
+  if (!lk || !scratch || scratch_bytes <= room) return;
+  const DeviceGuard g(device);
+  (void)hipFree(scratch);
+  scratch = nullptr;
+  scratch_bytes = 0;
+}
+
 // From two chunks on through the staging buffers: the card fills one while a thread empties
 // another into the caller's memory, whose fresh pages cost more than the copy.  A plain copy
 // runs at 10 GB/s into fresh pages; four threads take 4 MB in 0.28 ms against 0.59 (1 MB:
@@ -1150,11 +1160,11 @@ int run_sweep_graph(mbir_job* j, int outer, int inner, mbir_sweep_stats* st)
   const size_t slots = (size_t)nsteps * width;
   if (j->gsched.n < slots) {
     j->gsched.release();
-    HIP_TRY(j->gsched.alloc(slots));
+    HIP_TRY(j->gsched.alloc(*j->pool, slots));
   }
   if (j->ustat.n < slots) {  // statistics by padded slot (the descriptor changes: recapture)
     j->ustat.release();
-    HIP_TRY(j->ustat.alloc(slots));
+    HIP_TRY(j->ustat.alloc(*j->pool, slots));
     j->J.ustat = j->ustat.p;
   }
   const bool stale = stale0 || std::memcmp(&j->graph_J, &j->J, sizeof(DevJob)) != 0;
@@ -1278,11 +1288,11 @@ int run_batch(mbir_ctx* ctx, const std::vector<mbir_job*>& jobs, const int* oute
   }
   if (ctx->djobs.n < (size_t)n) {
     ctx->djobs.release();
-    HIP_TRY(ctx->djobs.alloc(n));
+    HIP_TRY(ctx->djobs.alloc(*ctx->pool, n));
   }
   if (ctx->ents.n < ent.size()) {
     ctx->ents.release();
-    HIP_TRY(ctx->ents.alloc(ent.size()));
+    HIP_TRY(ctx->ents.alloc(*ctx->pool, ent.size()));
   }
   hipStream_t s = ctx->stream;
   for (mbir_job* j : jobs) HIP_TRY(hipStreamSynchronize(j->stream));  // schedules uploaded

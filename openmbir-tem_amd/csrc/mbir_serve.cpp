@@ -189,12 +189,18 @@ void mbir_server::setup_loop()
     reserved = reserved - (uint64_t)r->reserved + (uint64_t)job->bytes;
     r->reserved = job->bytes;
     peak_reserved = std::max(peak_reserved, reserved);
+    // the setups' scratch, which the estimate covered, stays only where the budget has room
+    // (another setup that holds it now is charged for it)
+    const size_t room = budget > reserved ? (size_t)(budget - reserved) : 0;
     std::vector<double>().swap(r->angles);
     std::vector<float>().swap(r->counts);
     std::vector<float>().swap(r->init);
     ready.push_back(r);
     cv_run.notify_all();
     cv_setup.notify_all();
+    lk.unlock();
+    ctx->pool->trim(room);
+    lk.lock();
   }
 }
 
@@ -566,7 +572,7 @@ extern "C" int32_t mbir_server_create(mbir_ctx* ctx, const mbir_server_opts* o, 
   // default-priority streams, one per lane
   if (hipStreamCreate(&s->lane_stream[0]) != hipSuccess ||
       hipStreamCreate(&s->lane_stream[1]) != hipSuccess ||
-      s->djobs.alloc(s->max_jobs) != hipSuccess) {
+      s->djobs.alloc(*ctx->pool, s->max_jobs) != hipSuccess) {
     for (hipStream_t& q : s->lane_stream)
       if (q) (void)hipStreamDestroy(q);
     s->djobs.release();
