@@ -782,8 +782,10 @@ void build_schedule(mbir_job* j, bool drop_empty_steps)
   st.resize(w);
 }
 
-// The units of step k, a row class, as k_build_schedule writes them.
-static void fill_step(const mbir_job* j, int k, LineRef* out)
+// f(unit) for the units of step k, a row class, in the order in which k_build_schedule writes
+// them.
+template <class F>
+static void each_unit(const mbir_job* j, int k, F&& f)
 {
   const StepShape q = step_shape(j);
   const int zb = j->step_class[k] / q.S, c = j->step_class[k] % q.S;
@@ -792,7 +794,7 @@ static void fill_step(const mbir_job* j, int k, LineRef* out)
       const int z = q.row(zb, r, sl), pad = q.range(sl);
       if (z < 0) continue;
       for (int l = z * q.Nx + c; l < (z + 1) * q.Nx; l += q.S)
-        if (j->nnz_h[l] > 0) *out++ = LineRef{l, j->cptr_h[l], j->nnz_h[l], pad};
+        if (j->nnz_h[l] > 0) f(LineRef{l, j->cptr_h[l], j->nnz_h[l], pad});
     }
 }
 
@@ -801,7 +803,8 @@ const LineRef* step_refs(const mbir_job* j, int k, LineRef* buf)
 {
   if (j->step_ptr[k + 1] - j->step_ptr[k] > kInlineLines) return nullptr;
   if (!j->sched_h.empty()) return j->sched_h.data() + j->step_ptr[k];
-  fill_step(j, k, buf);
+  LineRef* at = buf;
+  each_unit(j, k, [&](const LineRef& r) { *at++ = r; });
   return buf;
 }
 
@@ -809,8 +812,9 @@ const LineRef* step_refs(const mbir_job* j, int k, LineRef* buf)
 void fill_schedule(mbir_job* j)
 {
   if (j->step_class.empty() || !j->sched_h.empty()) return;
-  j->sched_h.resize(j->units());
-  for (size_t k = 0; k + 1 < j->step_ptr.size(); ++k) fill_step(j, (int)k, j->sched_h.data() + j->step_ptr[k]);
+  j->sched_h.reserve(j->units());
+  for (size_t k = 0; k + 1 < j->step_ptr.size(); ++k)
+    each_unit(j, (int)k, [&](const LineRef& r) { j->sched_h.push_back(r); });
 }
 
 // The sweep's schedule into j->sched on stream s (the accumulators are formed from the
@@ -1609,16 +1613,20 @@ extern "C" int32_t mbir_job_get_schedule(mbir_job* job, int32_t* step_ptr, int32
   const int32_t steps = job->step_ptr.empty() ? 0 : (int32_t)job->step_ptr.size() - 1;
   if (step_ptr)
     for (int32_t k = 0; k <= steps && k <= cap_steps; ++k) step_ptr[k] = job->step_ptr[k];
-  if (units) {
-    fill_schedule(job);
-    const int64_t n = std::min<int64_t>((int64_t)job->sched_h.size(), cap_units);
-    for (int64_t i = 0; i < n; ++i) {
-      const LineRef& r = job->sched_h[i];
+  if (units) {  // worked out into the caller's array: the job is only read
+    int64_t i = 0;
+    auto put = [&](const LineRef& r) {
+      if (i >= cap_units) return;
       const int ny = r.pad >> 16;
       units[3 * i] = r.line;
       units[3 * i + 1] = ny ? (r.pad & 0xffff) : 0;
       units[3 * i + 2] = ny ? ny : job->g.N_y;
-    }
+      ++i;
+    };
+    if (job->step_class.empty())  // listed lines
+      for (const LineRef& r : job->sched_h) put(r);
+    else
+      for (int32_t k = 0; k < steps && i < cap_units; ++k) each_unit(job, k, put);
   }
   return steps;
 }

@@ -186,7 +186,8 @@ struct mbir_job {
   DevBuf<mbir::UnitStat> ustat;  // per schedule position: the unit's sweep statistics
   DevBuf<double> red;             // block sums of the statistics (5 kReduceBlocks)
   // the sweep's schedule: step k is row class step_class[k] (empty: listed lines, in
-  // sched_h), its units [step_ptr[k], step_ptr[k + 1]); sched_h is filled when asked for
+  // sched_h), its units [step_ptr[k], step_ptr[k + 1]); sched_h then holds the list only in a
+  // graph's sweeps (fill_schedule)
   std::vector<int> step_class, step_ptr;
   std::vector<int> class_n;   // units of every row class
   std::vector<int> steps_h;   // step_class and step_ptr as uploaded to `steps`
