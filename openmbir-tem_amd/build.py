@@ -46,6 +46,8 @@ SOURCES = [
     (os.path.join(ENGINE, "mbir_estimate.cpp"), ["-x", "c++"]),
 ]
 CLI = os.path.join(HERE, "engine_cli")
+# device-side comparisons of the GPU tests, linked against the library
+CHECKS = os.path.join(REPO, "tests", "native")
 
 
 def build(verbose=True):
@@ -69,6 +71,14 @@ def build(verbose=True):
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
     os.replace(CLI + ".tmp", CLI)
+    out = os.path.join(CHECKS, "libmbir_checks.so")
+    cmd = [HIPCC] + COMMON + ["-I", CSRC, "-x", "hip"] + DEVICE + [
+        os.path.join(CHECKS, "checks.hip"), "-shared", "-o", out + ".tmp", "-L", HERE, "-lmbir_tem",
+        "-Wl,-rpath,$ORIGIN/../../openmbir-tem_amd"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    os.replace(out + ".tmp", out)
     return OUT
 
 
