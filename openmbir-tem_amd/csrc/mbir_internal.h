@@ -212,8 +212,10 @@ hipError_t launch_detector_response(int N_theta, const VoxelProfile* prof, const
                                     double dxz, double delta_r, double offsetR, double* H,
                                     hipStream_t s);
 hipError_t launch_line_nnz(const DevJob& J, int* line_nnz, float* x, hipStream_t s);
-// out = the projection of vol (every entry written)
-hipError_t launch_forward_project(const DevJob& J, const float* vol, double* out, hipStream_t s);
+// out = the projection of vol (every entry written).  Volumes of wide_from voxels and more take
+// 64-bit line addresses (from 2^30 on byte offsets no longer fit 32 bits).
+hipError_t launch_forward_project(const DevJob& J, const float* vol, double* out, hipStream_t s,
+                                  uint64_t wide_from = 1ull << 30);
 hipError_t launch_init_error(const DevJob& J, const double* yest, hipStream_t s);
 // fine volume (sizes N_z, N_x, N_y) from the coarse one of sizes N/2, replicated 2 x 2 x 2;
 // lines with line_nnz 0 stay 0

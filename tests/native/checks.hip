@@ -140,3 +140,21 @@ extern "C" int checks_selector(int what, uint64_t seed, int per, unsigned long l
   (void)hipFree(d);
   return r == hipSuccess ? 0 : -1;
 }
+
+// The projection of vol by 64-bit line addresses, whatever the volume's size
+extern "C" int checks_project_wide(mbir_job* j, const float* vol, double* out)
+{
+  const size_t M = (size_t)j->g.N_theta * j->g.N_r * j->g.N_t;
+  const size_t V = (size_t)j->g.N_z * j->g.N_x * j->g.N_y;
+  float* dv = nullptr;
+  double* dout = nullptr;
+  hipError_t r = hipMalloc((void**)&dv, V * sizeof(float));
+  if (r == hipSuccess) r = hipMalloc((void**)&dout, M * sizeof(double));
+  if (r == hipSuccess) r = hipMemcpy(dv, vol, V * sizeof(float), hipMemcpyHostToDevice);
+  if (r == hipSuccess) r = launch_forward_project(j->J, dv, dout, j->stream, 0);
+  if (r == hipSuccess) r = hipStreamSynchronize(j->stream);
+  if (r == hipSuccess) r = hipMemcpy(out, dout, M * sizeof(double), hipMemcpyDeviceToHost);
+  if (dv) (void)hipFree(dv);
+  if (dout) (void)hipFree(dout);
+  return r == hipSuccess ? 0 : -1;
+}

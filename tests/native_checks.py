@@ -12,4 +12,5 @@ def load():
     capi.lib()  # the library whose functions the checks call
     lib = C.CDLL(PATH)
     lib.checks_selector.argtypes = [C.c_int, C.c_uint64, C.c_int, C.POINTER(C.c_ulonglong)]
+    lib.checks_project_wide.argtypes = [C.c_void_p, C.POINTER(C.c_float), C.POINTER(C.c_double)]
     return lib
