@@ -635,7 +635,6 @@ int setup_job(mbir_job* j)
     J.nx_div = (m < (1ull << 32) && lmax * r < (1ull << 32)) ? (uint32_t)m : 0u;
   }
   J.NB = NB;
-  J.nslots = NT * NB;
   J.vlr_max = 1;
   for (int c : vn) J.vlr_max = std::max(J.vlr_max, c);
   // the slices' rows are disjoint (checked above), so they cover the detector when they
@@ -651,7 +650,7 @@ int setup_job(mbir_job* j)
   J.spare_b = (uint32_t)(M * 4);
   J.x = j->x.p; J.e = j->e.p; J.y = j->y.p; J.wfull = nullptr; J.wview = j->wview.p;
   J.I0 = j->I0.p; J.mu = j->mu.p;
-  J.sched = j->sched.p; J.ustat = j->ustat.p;
+  J.ustat = j->ustat.p;
   // the error-sinogram update where a stream's values are not kept in registers: a
   // plain read-modify-write on conflict-free steps (no two lines of a step share a
   // detector bin; 12 % faster per launch than fp32 atomics on a 141-view 512x64x256
@@ -1910,7 +1909,6 @@ extern "C" int32_t mbir_job_set_volume(mbir_job* j, const float* vol)
 {
   if (!j || !vol) return MBIR_ERR_INPUT;
   const size_t V = (size_t)j->g.N_z * j->g.N_x * j->g.N_y;
-  const size_t M = (size_t)j->g.N_theta * j->g.N_r * j->g.N_t;
   hipStream_t s = j->stream;
   HIP_TRY(hipMemcpyAsync(j->x.p, vol, V * sizeof(float), hipMemcpyHostToDevice, s));
   return project_error(j, s);
@@ -1929,7 +1927,6 @@ extern "C" int32_t mbir_job_upsample_volume(mbir_job* fine, const mbir_job* coar
   if (c.N_z != f.N_z / 2 || c.N_x != f.N_x / 2 || c.N_y != f.N_y / 2 || c.N_z < 1 || c.N_x < 1 ||
       c.N_y < 1)
     return MBIR_ERR_INPUT;
-  const size_t M = (size_t)f.N_theta * f.N_r * f.N_t;
   hipStream_t s = fine->stream;
   HIP_TRY(hipStreamSynchronize(coarse->stream));  // the coarse volume is final
   HIP_TRY(launch_upsample2(coarse->x.p, fine->x.p, fine->line_nnz.p, f.N_z, f.N_x, f.N_y, s));

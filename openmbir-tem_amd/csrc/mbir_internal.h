@@ -112,7 +112,6 @@ struct DevJob {
                          // BF_OFFSET), spare row 0; null without
   // ---- the other kernels' ----
   int NB;                // slots (candidate detector bins) per view
-  int nslots;            // N_theta * NB
   int vlr_max;           // max detector rows of any slice (1 when delta_xy = delta_t)
   int rows_covered;      // 1: every detector row belongs to a slice
   int unit_max;          // slices of the job's longest schedule unit (N_y for whole lines):
@@ -122,7 +121,6 @@ struct DevJob {
   int held;              // 1: the register-held form of the line update applies (units of 9 to
                          // 64 slices, one detector row each, streams of at most 40 entries,
                          // plain or bright-field weights, conflict-free steps)
-  int pad_;
   double x0, z0, delta_xz, delta_r, R0, RMax, offsetR;
   double inv_delta_r, inv_offsetR;
   const double* cosv;    // [N_theta]
@@ -137,7 +135,6 @@ struct DevJob {
   const double* mu;      // [N_theta]
   double mrf_qd, mrf_cd, sigma_pd, sigma_pqd;
   double bragg_d, delta_d;  // T and delta in FP64 (cost, nuisance updates)
-  const LineRef* sched;  // [N_z * N_x * y slabs] units of the current sweep, step by step
 };
 
 
@@ -241,8 +238,6 @@ hipError_t launch_icd_batch_step(int ypl, int nv, const DevJob* jobs, const MixE
 hipError_t launch_build_columns(const DevJob& J, int* row, float* a, hipStream_t s);
 // the gain- and weight-folded column values, and the lines' theta2 factors kk
 hipError_t launch_column_weights(const DevJob& J, float* ka, float* kw, double* kk, hipStream_t s);
-hipError_t launch_export_column(const DevJob& J, int z, int x, float* vals, int* rows,
-                                hipStream_t s);
 // joint estimation / weights / cost (FP64)
 hipError_t launch_joint_sums(const DevJob& J, double* sums6, hipStream_t s);
 hipError_t launch_joint_solve(int N_theta, const double* sums6, double target_gain,
