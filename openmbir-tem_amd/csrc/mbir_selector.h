@@ -48,11 +48,11 @@ __device__ inline bool kept_by_root(float e, float aw, float T)
   return fabsf(e * sqrtf(aw)) < T;
 }
 
-// Whether e^2 aw against T^2 may decide it: T positive and its square not small enough to
-// lose bits (one that overflows leaves every entry near)
-__device__ inline bool square_decides(float T) { return T > kRejectLo; }
+// T^2, or not a number where the square may not decide: T not positive, or so small that the
+// squares lose bits (one that overflows leaves every entry near)
+__device__ inline float square_of(float T) { return T > kRejectLo ? T * T : NAN; }
 
-// The selector by e^2 aw < T2 = T^2; near is set where the two lie within 2e-6 of each other
+// The selector by e^2 aw < T2 = square_of(T); near is set where the two lie within 2e-6 of each other
 // (or are not numbers) and kept_by_root has to decide.  The squares are off by three
 // roundings and |e sqrt(aw)| by two, 4.2e-7 of T2 in all.
 __device__ inline bool kept_by_square(float e, float aw, float T2, bool& near)

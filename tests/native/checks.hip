@@ -105,9 +105,8 @@ __global__ void k_selector(uint64_t seed, int per, unsigned long long* out)
     const float y = fabsf(e * sqrtf(w));
     const float T = hash(s) & 7 ? __uint_as_float(__float_as_uint(y) + hash(s) % 129 - 64)
                                 : draw(s, -49, 70);
-    if (!square_decides(T)) continue;
     bool near = false;
-    const bool kept = kept_by_square(e, w, T * T, near);
+    const bool kept = kept_by_square(e, w, square_of(T), near);
     if (near) continue;
     ++n;
     bad += kept != kept_by_root(e, w, T);
