@@ -145,7 +145,8 @@ struct DeviceGuard {
 
 mbir_pool::~mbir_pool()
 {
-  if (!scratch && !stage) return;
+  // (the events are made first: they may be there without the staging memory)
+  if (!scratch && !stage && !ev[0]) return;
   const DeviceGuard g(device);
   if (scratch) (void)hipFree(scratch);
   if (stage) (void)hipHostFree(stage);
