@@ -709,6 +709,8 @@ int setup_job(mbir_job* j)
     while (ty < J.unit_max && ty < 64) ty <<= 1;
     const int streams = kIcdWaves * (64 / ty);
     J.batch = ((nmax + streams - 1) / streams + 3) & ~3;
+    // (batches of up to 40 entries, 148 views in units of 33 to 64 slices, are compiled and
+    // measured; longer ones would fit the single-job kernel's registers)
     J.held = umin > 8 && J.unit_max <= 64 && J.vlr_max <= 1 && !J.bfs && !J.e_atomic &&
              g.N_t < 65536 && J.batch <= 40;
   }

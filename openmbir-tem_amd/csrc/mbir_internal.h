@@ -183,7 +183,11 @@ struct TickArgs {
 
 // Choice between the two forms of the batched line kernels (identical results):
 // 1 = prefetching (shorter line latency), 0 = without prefetch (fewer registers), per
-// kernel shape (ypl 1|2, nv 1|2) and launch size (workgroups) bucket.
+// kernel shape (ypl 1|2, nv 1|2) and launch size (workgroups) bucket.  Without a measurement
+// of the caller's jobs: prefetching up to 512 (26.6 ns per workgroup against 28.6 at about
+// 350 on jobs of one shape, 23.1 against 24.6 at 520 to 600, 19.3 against 18.4 at about
+// 1000: the crossing lies inside the third bucket, which as a whole takes the other form; on
+// a mix of slab jobs that form is ahead over all of it, 26.1 against 29.7).
 constexpr int kTuneBuckets = 5;
 inline int tune_bucket(int nwg)
 {
