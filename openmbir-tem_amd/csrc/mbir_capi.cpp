@@ -195,6 +195,15 @@ void mbir_pool::trim(size_t room)
   scratch_bytes = 0;
 }
 
+// Device memory (a plain copy reaches it, whatever the direction it names)
+static bool on_device(const void* p)
+{
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeDevice;
+  (void)hipGetLastError();  // memory that the runtime does not know
+  return false;
+}
+
 // From two chunks on through the staging buffers: the card fills one while a thread empties
 // another into the caller's memory, whose fresh pages cost more than the copy.  A plain copy
 // runs at 10 GB/s into fresh pages; four threads take 4 MB in 0.28 ms against 0.59 (1 MB:
@@ -203,7 +212,7 @@ void mbir_pool::trim(size_t room)
 hipError_t mbir_pool::copy_out(void* dst, const void* src, size_t bytes, hipStream_t s)
 {
   std::unique_lock<std::mutex> lk(stage_mu, std::defer_lock);
-  if (bytes < 2 * kCopyChunk || !lk.try_lock() || make_stage() != hipSuccess) {
+  if (bytes < 2 * kCopyChunk || on_device(dst) || !lk.try_lock() || make_stage() != hipSuccess) {
     const hipError_t r = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
     return r != hipSuccess ? r : hipStreamSynchronize(s);
   }

@@ -47,7 +47,8 @@ struct mbir_pool {
   // gives the scratch block back if it is larger than `room` and no call uses it (a call that
   // does is charged for it elsewhere, and its end is the time to ask again)
   void trim(size_t room);
-  // dst = src (device) of stream s, in host memory when it returns
+  // dst = src (device) of stream s, there when it returns (dst: host memory; device memory is
+  // taken too, as a plain copy does)
   hipError_t copy_out(void* dst, const void* src, size_t bytes, hipStream_t s);
   ~mbir_pool();
 };
